@@ -1,0 +1,33 @@
+"""CPU: the rules that choose between kernels and launch shapes (csrc/routes.h),
+compiled by the host compiler, at the sizes where the measured lines lie."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "vulkanhybridraytracer_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    """rule("expression") -> the values of C++ expressions over namespace hr"""
+    tmp = tmp_path_factory.mktemp("routes")
+
+    def run(*exprs):
+        src = tmp / "t.cpp"
+        src.write_text('#include <cstdio>\n#include "routes.h"\nusing namespace hr;\nint main() {\n'
+                       + "".join('  printf("%%llu\\n", (unsigned long long)(%s));\n' % e for e in exprs)
+                       + "  return 0;\n}\n")
+        subprocess.check_call(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(src), "-o", str(tmp / "t")])
+        return [int(v) for v in subprocess.check_output([str(tmp / "t")]).split()]
+    return run
+
+
+def test_dealt_queue_walks_with_part_of_its_own_lanes(rule):
+    """a wave leaves the node loop for its leaves only when a share of the lanes
+    it holds has one, also where it holds few"""
+    lanes = list(range(1, 65))
+    below = rule(*["queue_leave_below(true, %du)" % n for n in lanes])
+    for n, b in zip(lanes, below):
+        assert b <= n - n // 4 and (n < 4 or b >= n // 2), (n, b)
+    assert rule("queue_leave_below(false, 64u)", "queue_leave_below(false, 20u)") == [16, 16]

@@ -13,7 +13,8 @@ LIB = os.path.join(HERE, "libhr.so")
 SOURCES = ["csrc/lbvh.hip", "csrc/trace.hip", "csrc/wavefront.hip", "csrc/denoise.hip", "csrc/temporal.hip",
            "csrc/gbuffer_io.hip", "csrc/rt.hip", "csrc/hr_api.hip", "csrc/dn_api.hip",
            "csrc/image_io.cpp", "csrc/assets.cpp"]  # the .cpp files are host-only (asset ingest)
-HEADERS = ["csrc/device_math.h", "csrc/internal.h", "csrc/trace_common.h", "csrc/api_internal.h", "csrc/image_io.h"]
+HEADERS = ["csrc/device_math.h", "csrc/internal.h", "csrc/trace_common.h", "csrc/api_internal.h", "csrc/image_io.h",
+           "csrc/routes.h"]
 LIBS = ["-lz"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
          "-fhip-fp32-correctly-rounded-divide-sqrt", "-Xclang", "-target-feature", "-Xclang",

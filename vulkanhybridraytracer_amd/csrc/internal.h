@@ -7,6 +7,7 @@
 #include <string>
 
 #include "hr/hr.h"
+#include "routes.h"
 
 namespace hr {
 

@@ -53,11 +53,10 @@ constexpr uint32_t DONE = 0xFFFFFFFFu;  // no node: no leaf code reaches it (few
 // The inner traversal loops also end when fewer lanes than this would keep
 // walking, so lanes whose ray ended or that hold two leaves get back to work
 // (leaf tests, new rays) instead of idling; results do not depend on it.
-// consume_rays (queues of closest-hit and hit-shadow rays) and item_loop
-// (sample-parallel shadow items) have their own. The item loop refills early:
-// lanes that start their rays together walk the same nodes, which a
-// wave-uniform node step reads through the scalar cache.
-constexpr int REFILL_MIN_LANES = 16;
+// consume_rays (queues of closest-hit and hit-shadow rays, queue_leave_below)
+// and item_loop (sample-parallel shadow items) have their own. The item loop
+// refills early: lanes that start their rays together walk the same nodes,
+// which a wave-uniform node step reads through the scalar cache.
 constexpr int REFILL_MIN_ITEMS = 56;
 
 // Node and triangle arrays live in global memory; reading them through
@@ -685,6 +684,7 @@ __device__ __forceinline__ void consume_queue(const DevScene& S, uint32_t n, uin
             cur = S.node_count ? 0u : DONE;
             continue;
         }
+        const uint32_t leave = queue_leave_below(DEALT, (uint32_t)__popcll(__ballot(1)));
         while (!COUNT && cur < LEAF_BIT) {
             cur = wide_step<STACK_CAP>(S.nodes4, cur, r, tmin, tbest, lds, spill, sp, c);
             // any hit: postpone the first leaf found and keep walking until
@@ -699,7 +699,7 @@ __device__ __forceinline__ void consume_queue(const DevScene& S, uint32_t n, uin
                     cur = sp < (int)STACK_LDS ? lds[sp * BLOCK] : spill[sp - STACK_LDS];
                 }
             }
-            if (__ballot(leaf == 0u) == 0ull || __popcll(__ballot(cur < LEAF_BIT)) < REFILL_MIN_LANES) break;
+            if (__ballot(leaf == 0u) == 0ull || (uint32_t)__popcll(__ballot(cur < LEAF_BIT)) < leave) break;
         }
         while (COUNT && cur < LEAF_BIT) {
             const float4* np = reinterpret_cast<const float4*>(S.nodes + cur);
