@@ -31,3 +31,11 @@ def test_dealt_queue_walks_with_part_of_its_own_lanes(rule):
     for n, b in zip(lanes, below):
         assert b <= n - n // 4 and (n < 4 or b >= n // 2), (n, b)
     assert rule("queue_leave_below(false, 64u)", "queue_leave_below(false, 20u)") == [16, 16]
+
+
+def test_adaptive_frames_of_few_samples_take_a_lane_per_group(rule):
+    """1 sample always, 2 in small scenes; other counts that are no power of two never go in stages"""
+    cases = [(1, 20_000, 0), (1, 4_000_000, 0), (2, 20_000, 0), (2, 99_999, 0), (2, 262_144, 1), (2, 4_000_000, 1),
+             (3, 4_000_000, 0), (4, 100, 1), (16, 20_000, 1), (48, 20_000, 0), (64, 1_000_000, 1), (65, 1_000_000, 0),
+             (128, 1_000_000, 0), (0, 1_000_000, 0)]
+    assert rule(*["adaptive_stages(%du, %du)" % (s, t) for s, t, _ in cases]) == [e for _, _, e in cases]

@@ -430,7 +430,7 @@ uint32_t make_jobs(const hr_context* ctx, const std::vector<FramePlan>& plans, s
 }
 
 // The sample-parallel shadow kernels take timed frames of 1 to 64 samples (with
-// adaptive sampling powers of two), all adaptive or none. Items are spaced by
+// adaptive sampling those of adaptive_stages), all adaptive or none. Items are spaced by
 // the largest count, so frames with 1-3 samples or no power of two join only
 // when the counts are within a factor of two; such frames can also go without
 // the scratch (spare), through the group-per-lane kernel that takes all other
@@ -450,7 +450,7 @@ SplPlan plan_spl(const FramePlan* plans, size_t nplans, uint32_t ngroups) {
         const FrameArgs& f = plans[i].f;
         const uint32_t S = f.samples;
         const bool pow2 = (S & (S - 1u)) == 0u;
-        if (plans[i].count || S < 1u || S > 64u || (f.adaptive && !pow2)) return sp;
+        if (plans[i].count || S < 1u || S > 64u || (f.adaptive && !adaptive_stages(S, plans[i].scene->ntri))) return sp;
         if (i > 0 && (f.adaptive != 0u) != sp.adaptive) return sp;
         sp.adaptive = f.adaptive != 0u;
         sp.spare = sp.spare || S < 4u || !pow2;

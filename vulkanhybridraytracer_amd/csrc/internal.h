@@ -170,7 +170,7 @@ struct ShadowJob {
 uint32_t shadow_groups(const FrameArgs& f, uint32_t tile_w);
 // writes `job` to device memory at dst (16-byte aligned) from a kernel argument
 hipError_t launch_store_job(const ShadowJob& job, ShadowJob* dst, hipStream_t st);
-// Frames with sample counts in 1..64 (adaptive sampling: powers of two), all
+// Frames with sample counts in 1..64 (adaptive sampling: adaptive_stages), all
 // adaptive or none: one lane per (group, sample) item, max_samples the largest
 // count. scratch: device memory of shadows_spl_scratch() bytes (0 where
 // shadows_spl_direct).

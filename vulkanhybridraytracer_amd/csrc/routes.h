@@ -27,4 +27,22 @@ namespace hr {
 //   1280 x 720, 1M triangles   4448 / 3467 / 3303
 HR_RULE uint32_t queue_leave_below(bool dealt, uint32_t live) { return dealt ? live * 3u / 4u : 16u; }
 
+// Triangles from which a scene's rays are long: they visit many nodes and their
+// data leaves the caches, so idle lanes and single launches cost less than walks
+// that wait for one another.
+constexpr uint32_t LARGE_SCENE = 100000u;
+
+// Adaptive shadow passes in stages over the listed groups (powers of two up to
+// 64), or a lane per group? With 1 or 2 samples there is one stage and nothing to
+// adapt, so the probes over all groups, 4 items each, and the lists are overhead:
+// us in stages and a lane per group, 2 lights in 20k triangles (spheres): 1
+// sample 256 x 256 218, 72, 1280 x 720 667, 198, 2 samples 667, 198; 4 lights in
+// 1M triangles: 1 sample 960 x 540 772, 573, but 2 samples 640 x 360 507, 791
+// and 1920 x 1080 1660, 2453 (262k: 480, 581 and 1372, 1817; 16k: 432, 412 and
+// 950, 1068).
+HR_RULE bool adaptive_stages(uint32_t samples, uint32_t tris) {
+    return samples >= 1u && samples <= 64u && (samples & (samples - 1u)) == 0u &&
+           (samples >= 4u || (samples == 2u && tris >= LARGE_SCENE));
+}
+
 }  // namespace hr
