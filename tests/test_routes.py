@@ -39,3 +39,24 @@ def test_adaptive_frames_of_few_samples_take_a_lane_per_group(rule):
              (3, 4_000_000, 0), (4, 100, 1), (16, 20_000, 1), (48, 20_000, 0), (64, 1_000_000, 1), (65, 1_000_000, 0),
              (128, 1_000_000, 0), (0, 1_000_000, 0)]
     assert rule(*["adaptive_stages(%du, %du)" % (s, t) for s, t, _ in cases]) == [e for _, _, e in cases]
+
+
+def test_shadow_routes_of_few_samples(rule):
+    """the measured fastest route of frames (samples, groups, triangles) at both sides of every line, and
+    the routes without memory for lists"""
+    def groups(w, h, lights):
+        return -(-w // 8) * -(-h // 8) * 64 * lights
+    group, once, direct, listed = 0, 1, 2, 3
+    cases = [((3, 0, groups(256, 256, 2), 20_482, 1), once), ((4, 0, groups(160, 100, 4), 16_384, 1), once),
+             ((2, 0, groups(640, 360, 2), 20_482, 1), once), ((1, 0, groups(960, 540, 2), 20_482, 1), once),
+             ((1, 0, groups(1280, 720, 2), 20_482, 1), listed), ((2, 0, groups(1920, 1080, 2), 20_482, 1), listed),
+             ((5, 0, groups(97, 64, 2), 20_482, 1), listed), ((1, 0, groups(97, 64, 4), 262_144, 1), listed),
+             ((1, 0, groups(1280, 720, 4), 262_144, 1), direct), ((2, 0, groups(1920, 1080, 4), 262_144, 1), direct),
+             ((2, 0, groups(1920, 1080, 4), 16_384, 1), listed), ((1, 0, groups(1920, 1080, 4), 16_384, 1), direct),
+             ((1, 0, groups(640, 360, 4), 1_048_576, 1), listed), ((1, 0, groups(1920, 1080, 4), 1_048_576, 1), listed),
+             ((2, 1, groups(1920, 1080, 4), 1_048_576, 1), listed), ((64, 1, groups(97, 64, 4), 20_482, 1), listed),
+             ((1, 0, groups(640, 360, 4), 1_048_576, 0), direct), ((2, 0, groups(97, 64, 4), 1_048_576, 0), once),
+             ((3, 0, groups(640, 360, 4), 1_048_576, 0), group), ((2, 1, groups(640, 360, 4), 1_048_576, 0), group),
+             ((3, 0, groups(97, 64, 4), 16_384, 0), once)]
+    got = rule(*["(unsigned)shadow_route(%du, %d, %du, %du, %d)" % a for a, _ in cases])
+    assert got == [e for _, e in cases]

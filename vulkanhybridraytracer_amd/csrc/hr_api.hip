@@ -433,14 +433,18 @@ uint32_t make_jobs(const hr_context* ctx, const std::vector<FramePlan>& plans, s
 // adaptive sampling those of adaptive_stages), all adaptive or none. Items are spaced by
 // the largest count, so frames with 1-3 samples or no power of two join only
 // when the counts are within a factor of two; such frames can also go without
-// the scratch (spare), through the group-per-lane kernel that takes all other
-// frames.
+// the scratch (spare). The group-per-lane kernel takes all other frames.
 struct SplPlan {
-    bool use = false;
+    ShadowRoute route = ShadowRoute::Group;
     bool adaptive = false;
     bool spare = false;
     uint32_t samples = 0;  // the largest count
+    uint32_t groups = 0, tris = 0;  // of all frames; of the largest scene
     size_t scratch = 0;
+    void choose(bool with_scratch) {
+        route = shadow_route(samples, adaptive, groups, tris, with_scratch);
+        scratch = route == ShadowRoute::Listed ? shadows_spl_scratch(groups, samples, adaptive) : 0;
+    }
 };
 
 SplPlan plan_spl(const FramePlan* plans, size_t nplans, uint32_t ngroups) {
@@ -454,36 +458,35 @@ SplPlan plan_spl(const FramePlan* plans, size_t nplans, uint32_t ngroups) {
         if (i > 0 && (f.adaptive != 0u) != sp.adaptive) return sp;
         sp.adaptive = f.adaptive != 0u;
         sp.spare = sp.spare || S < 4u || !pow2;
+        sp.tris = std::max(sp.tris, plans[i].scene->ntri);
         smax = std::max(smax, S);
         smin = std::min(smin, S);
     }
     if (sp.spare && smax > 2u * smin) return sp;
-    uint32_t lg2s = 0;
-    while ((1u << lg2s) < smax) ++lg2s;
-    if (((uint64_t)ngroups << lg2s) >= (1ull << 32)) return sp;
+    if (((uint64_t)ngroups << log2_up(smax)) >= (1ull << 32)) return sp;
     sp.samples = smax;
-    sp.scratch = shadows_spl_scratch(ngroups, smax, sp.adaptive);
-    sp.use = true;
+    sp.groups = ngroups;
+    sp.choose(true);
     return sp;
 }
 // ... with its scratch in ctx->work
 hr_status plan_spl_work(hr_context* ctx, const FramePlan* plans, size_t nplans, uint32_t ngroups, SplPlan& sp) {
     sp = plan_spl(plans, nplans, ngroups);
-    if (!sp.use) return HR_OK;
+    if (sp.route != ShadowRoute::Listed) return HR_OK;
     bool oom = false;
     HR_TRY(ensure_work(ctx, sp.scratch, sp.spare ? &oom : nullptr));
-    if (oom) sp = SplPlan{};
+    if (oom) sp.choose(false);
     return HR_OK;
 }
 
 // Kernels of a shadow pass (device jobs already uploaded); scratch holds
-// sp.scratch bytes when sp.use.
+// sp.scratch bytes.
 // (wide_count: the 4-wide nodes of the first frame's scene; used for one frame)
 hr_status enqueue_shadows(hr_context* ctx, const ShadowJob* d_jobs, uint32_t n, uint32_t ngroups, const SplPlan& sp,
                           bool count, uint32_t* next_group, uint32_t* scratch, uint32_t wide_count) {
-    if (sp.use)
-        HR_HIP(ctx, launch_shadows_spl(d_jobs, n, ngroups, sp.samples, sp.adaptive, ctx->d_counters, ctx->stream,
-                                       next_group, scratch, ctx->resident_blocks, wide_count));
+    if (sp.route != ShadowRoute::Group)
+        HR_HIP(ctx, launch_shadows_spl(sp.route, d_jobs, n, ngroups, sp.samples, sp.adaptive, ctx->d_counters,
+                                       ctx->stream, next_group, scratch, ctx->resident_blocks, wide_count));
     else
         HR_HIP(ctx, launch_shadows(d_jobs, n, ngroups, ctx->d_counters, count, ctx->stream, next_group,
                                    ctx->resident_blocks));
@@ -1102,8 +1105,8 @@ hr_status hr_trace_shadows_noalloc(hr_scene* s, const hr_gbuffer* gb, const hr_l
     ShadowJob job;
     const uint32_t ngroups = fill_job(ctx, fp, 0u, job);
     SplPlan sp = plan_spl(&fp, 1, ngroups);
-    if (sp.spare && NOALLOC_BITS_OFFSET + sp.scratch > NOALLOC_BYTES) sp = SplPlan{};
-    const size_t need = NOALLOC_BITS_OFFSET + (sp.use ? sp.scratch : 0);
+    if (sp.spare && NOALLOC_BITS_OFFSET + sp.scratch > NOALLOC_BYTES) sp.choose(false);
+    const size_t need = NOALLOC_BITS_OFFSET + sp.scratch;
     if (need > NOALLOC_BYTES)
         return fail(ctx, HR_E_UNSUPPORTED, "the frame needs %zu bytes of scratch, above HR_NOALLOC_SCRATCH_BYTES (%zu)",
                     need, NOALLOC_BYTES);
@@ -1336,7 +1339,7 @@ hr_status hr_graph_capture(hr_context* ctx, const hr_frame_desc* frames, uint32_
     SplPlan sp = plan_spl(plans.data(), plans.size(), ngroups);
     auto need = [&](uint32_t b) {
         size_t bytes = batch_work_bytes(ctx, plans, b);
-        return (bytes != 0 && sp.use && sp.scratch > bytes) ? sp.scratch : bytes;
+        return (bytes != 0 && sp.scratch > bytes) ? sp.scratch : bytes;
     };
     uint32_t mb = ctx->tuning.wave_budget_mb;
     if (need(mb) == 0) return fail(ctx, HR_E_UNSUPPORTED, "reflection slab too large");
@@ -1355,11 +1358,11 @@ hr_status hr_graph_capture(hr_context* ctx, const hr_frame_desc* frames, uint32_
             return fail(ctx, HR_E_UNSUPPORTED, "reflection slab too large");
         }
         e = hipMalloc(&g->work, bytes);
-        if (e != hipErrorOutOfMemory || (mb <= 64u && !(sp.use && sp.spare))) break;
+        if (e != hipErrorOutOfMemory || (mb <= 64u && !(sp.scratch && sp.spare))) break;
         (void)hipGetLastError();
         g->work = nullptr;
         e = hipSuccess;
-        if (mb <= 64u) sp = SplPlan{};  // the shadow pass without scratch
+        if (mb <= 64u) sp.choose(false);  // the shadow pass without scratch
         mb = mb / 2u < 64u ? 64u : mb / 2u;
     }
     if (e == hipSuccess) e = hipMemcpy(g->d_jobs, jobs.data(), n * sizeof(ShadowJob), hipMemcpyHostToDevice);

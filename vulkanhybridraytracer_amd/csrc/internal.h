@@ -145,13 +145,6 @@ enum : int {
 // to one cache line serialise.
 constexpr uint32_t C_STRIDE = 32;
 
-// A launch of `packets` waves that walk the tree once per wave (packet_walk)
-// waits for its nodes one after another and hides that only behind other
-// waves: at 640 x 360 (3,600 packets) the primary rays took 127 us as packets
-// and 88 us with a walk per lane, at 1280 x 720 and above (14,400) packets win.
-constexpr uint32_t PACKETS_MIN = 8192u;
-inline bool packets_fill(uint64_t packets) { return packets >= PACKETS_MIN; }
-
 // ---- launchers (trace.hip) ---------------------------------------------------
 hipError_t launch_gbuffer(const DevScene& s, const FrameArgs& f, GBufView gb, unsigned long long* counters,
                           bool count, hipStream_t st);
@@ -172,14 +165,13 @@ uint32_t shadow_groups(const FrameArgs& f, uint32_t tile_w);
 hipError_t launch_store_job(const ShadowJob& job, ShadowJob* dst, hipStream_t st);
 // Frames with sample counts in 1..64 (adaptive sampling: adaptive_stages), all
 // adaptive or none: one lane per (group, sample) item, max_samples the largest
-// count. scratch: device memory of shadows_spl_scratch() bytes (0 where
-// shadows_spl_direct).
-bool shadows_spl_direct(uint32_t max_samples, bool adaptive);
+// count, by the route Once, Direct or Listed. scratch: for Listed, device memory
+// of shadows_spl_scratch() bytes.
 size_t shadows_spl_scratch(uint32_t ngroups, uint32_t max_samples, bool adaptive);
 // wide_count: the 4-wide nodes of a single frame's scene (to choose 32-bit
 // node addressing), ignored for several frames
-hipError_t launch_shadows_spl(const ShadowJob* jobs_dev, uint32_t njobs, uint32_t ngroups, uint32_t max_samples,
-                              bool adaptive, unsigned long long* counters, hipStream_t st, uint32_t* next_item,
+hipError_t launch_shadows_spl(ShadowRoute route, const ShadowJob* jobs_dev, uint32_t njobs, uint32_t ngroups,
+                              uint32_t max_samples, bool adaptive, unsigned long long* counters, hipStream_t st, uint32_t* next_item,
                               uint32_t* scratch, uint32_t resident_blocks, uint32_t wide_count);
 // jobs_dev: njobs ShadowJob in device memory; next_group: BAND_COUNTER_BYTES
 // of device memory holding the SHADOW_QUEUES band counters, BAND_STRIDE words

@@ -45,4 +45,60 @@ HR_RULE bool adaptive_stages(uint32_t samples, uint32_t tris) {
            (samples >= 4u || (samples == 2u && tris >= LARGE_SCENE));
 }
 
+// A launch of `packets` waves that walk the tree once per wave (packet_walk)
+// waits for its nodes one after another and hides that only behind other
+// waves: at 640 x 360 (3,600 packets) the primary rays took 127 us as packets
+// and 88 us with a walk per lane, at 1280 x 720 and above (14,400) packets win.
+constexpr uint32_t PACKETS_MIN = 8192u;
+HR_RULE bool packets_fill(uint64_t packets) { return packets >= PACKETS_MIN; }
+
+// How a shadow pass of 1 to 64 samples runs. Items: one per group (pixel and
+// light) and sample, 2^lg2s >= samples to a group, 64 to a wave.
+enum class ShadowRoute : uint32_t {
+    Group,   // a lane per group, its samples one after the other (k_shadows)
+    Once,    // a lane per item and walk, all groups (k_shadows_once)
+    Direct,  // packets of items, all groups (k_shadows_direct)
+    Listed,  // the groups that need rays listed, their items traced (k_shadows_spl)
+};
+HR_RULE uint32_t log2_up(uint32_t n) {
+    uint32_t l = 0u;
+    while ((1u << l) < n) ++l;
+    return l;
+}
+// Listing the groups costs about 30 us of launches, and drops 57% of the items of
+// the terrain scenes' 1080p frames. Without adaptive sampling, us of Group, Once,
+// Direct, Listed (Direct was taken from 8192 waves of items on, Once below):
+//                                  waves
+//   20k triangles (spheres, 2 lights)
+//     256 x 256, 3 samples          8,192    129   92  149  165
+//     640 x 360, 2 samples         14,400    188  145  186  190
+//     960 x 540, 1 sample          16,320    187  171  198  201
+//     1280 x 720, 1 sample         28,800    209  243  222  222
+//     1920 x 1080, 2 samples      129,600    387  883  420  363
+//   16k triangles (terrain, 4 lights)
+//     160 x 100, 4 samples          4,160    392  144  132  176
+//     400 x 300, 2 samples         15,200    376  253  282  246
+//     1920 x 1080, 1 sample       129,600    706  990  496  564
+//     1920 x 1080, 2 samples      259,200   1053 1885  766  670
+//   262k triangles
+//     97 x 64, 1 sample               416    163  172  340  134
+//     640 x 360, 1 sample          14,400    332  346  373  275
+//     1280 x 720, 1 sample         57,600    629  760  456  475
+//     1920 x 1080, 2 samples      259,200   1840 2390 1035 1190
+//   1M triangles
+//     256 x 256, 1 sample           4,096    352  312  604  230
+//     640 x 360, 1 sample          14,400    434  428  584  292
+//     1920 x 1080, 1 sample       129,600   1358 1644 1020  939
+// scratch: is there memory for the lists?
+HR_RULE ShadowRoute shadow_route(uint32_t samples, bool adaptive, uint32_t groups, uint32_t tris, bool scratch) {
+    const uint64_t waves = ((uint64_t)groups << log2_up(samples)) >> 6;
+    if (!adaptive && samples <= 4u && tris < LARGE_SCENE && waves < 16384u) return ShadowRoute::Once;
+    if (!adaptive && samples == 1u && tris < 500000u && waves >= 49152u) return ShadowRoute::Direct;
+    if (!adaptive && samples == 2u && tris >= LARGE_SCENE && tris < 500000u && waves >= 98304u)
+        return ShadowRoute::Direct;
+    if (scratch) return ShadowRoute::Listed;
+    if (adaptive || samples > 2u) return ShadowRoute::Group;
+    return packets_fill(waves) ? ShadowRoute::Direct : ShadowRoute::Once;
+}
+
 }  // namespace hr
