@@ -438,6 +438,7 @@ struct SplPlan {
     ShadowRoute route = ShadowRoute::Group;
     bool adaptive = false;
     bool spare = false;
+    bool scattered = false;
     uint32_t samples = 0;  // the largest count
     uint32_t groups = 0, tris = 0;  // of all frames; of the largest scene
     size_t scratch = 0;
@@ -458,6 +459,7 @@ SplPlan plan_spl(const FramePlan* plans, size_t nplans, uint32_t ngroups) {
         if (i > 0 && (f.adaptive != 0u) != sp.adaptive) return sp;
         sp.adaptive = f.adaptive != 0u;
         sp.spare = sp.spare || S < 4u || !pow2;
+        sp.scattered = sp.scattered || scattered_lights(f);
         sp.tris = std::max(sp.tris, plans[i].scene->ntri);
         smax = std::max(smax, S);
         smin = std::min(smin, S);
@@ -486,7 +488,8 @@ hr_status enqueue_shadows(hr_context* ctx, const ShadowJob* d_jobs, uint32_t n, 
                           bool count, uint32_t* next_group, uint32_t* scratch, uint32_t wide_count) {
     if (sp.route != ShadowRoute::Group)
         HR_HIP(ctx, launch_shadows_spl(sp.route, d_jobs, n, ngroups, sp.samples, sp.adaptive, ctx->d_counters,
-                                       ctx->stream, next_group, scratch, ctx->resident_blocks, wide_count));
+                                       ctx->stream, next_group, scratch, ctx->resident_blocks, wide_count, sp.tris,
+                                       sp.scattered));
     else
         HR_HIP(ctx, launch_shadows(d_jobs, n, ngroups, ctx->d_counters, count, ctx->stream, next_group,
                                    ctx->resident_blocks));

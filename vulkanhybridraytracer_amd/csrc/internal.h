@@ -117,6 +117,14 @@ struct FrameArgs {
     uint32_t adaptive;  // HR_FLAG_ADAPTIVE
     uint32_t unorm8;    // UNORM8_SHADOW | UNORM8_LIT: the reference's 8-bit image formats
 };
+// do a light's rays from one point scatter (a disk of some radius)?
+inline bool scattered_lights(const FrameArgs& f) {
+    for (uint32_t i = 0; i < f.nl; ++i) {
+        const bool rect = f.has_shapes && f.shapes[i].type == HR_LIGHT_RECT && !(f.lights[i].pos_maxdist[3] < 0.0f);
+        if (!rect && f.lights[i].radius != 0.0f) return true;
+    }
+    return false;
+}
 constexpr uint32_t UNORM8_SHADOW = 1u;  // shadow buffers are R8_UNORM
 constexpr uint32_t UNORM8_LIT = 2u;     // lit is B8G8R8A8_UNORM
 
@@ -168,11 +176,13 @@ hipError_t launch_store_job(const ShadowJob& job, ShadowJob* dst, hipStream_t st
 // count, by the route Once, Direct or Listed. scratch: for Listed, device memory
 // of shadows_spl_scratch() bytes.
 size_t shadows_spl_scratch(uint32_t ngroups, uint32_t max_samples, bool adaptive);
-// wide_count: the 4-wide nodes of a single frame's scene (to choose 32-bit
-// node addressing), ignored for several frames
+// wide_count, tris: the 4-wide nodes (to choose 32-bit node addressing) and
+// triangles of a single frame's scene, ignored for several frames; scattered:
+// scattered_lights of any frame
 hipError_t launch_shadows_spl(ShadowRoute route, const ShadowJob* jobs_dev, uint32_t njobs, uint32_t ngroups,
                               uint32_t max_samples, bool adaptive, unsigned long long* counters, hipStream_t st, uint32_t* next_item,
-                              uint32_t* scratch, uint32_t resident_blocks, uint32_t wide_count);
+                              uint32_t* scratch, uint32_t resident_blocks, uint32_t wide_count, uint32_t tris,
+                              bool scattered);
 // jobs_dev: njobs ShadowJob in device memory; next_group: BAND_COUNTER_BYTES
 // of device memory holding the SHADOW_QUEUES band counters, BAND_STRIDE words
 // apart (reset by the launch); resident_blocks: the persistent grid size

@@ -101,4 +101,31 @@ HR_RULE ShadowRoute shadow_route(uint32_t samples, bool adaptive, uint32_t group
     return packets_fill(waves) ? ShadowRoute::Direct : ShadowRoute::Once;
 }
 
+// The number of waves of listed items, `samples` per (surface point, light), from
+// which they are traced as packets (packet_loop) and not with a walk per lane
+// (item_loop). Packets need waves to hide their serial node loads behind, and
+// rays that stay together: rays of one point do, those of neighbouring points
+// less the more triangles lie between them, and less to a disk light (random
+// directions: scattered) than to an area light (stratified). us per lane and as packets
+// (waves with rays), area lights:
+//   262k triangles  640 x 360  4 samples 411, 405 (28,700), 8 samples 575, 509
+//                              (57,400), 16 samples 878, 674 (115,000)
+//   1M              256 x 256  16 samples 452, 390 (29,600); 640 x 360 4 samples
+//                              498, 540 (22,500), 8 samples 671, 589 (45,100)
+//   4M              256 x 256  16 samples 608, 517 (33,100); 640 x 360 8 samples
+//                              854, 891 (49,900); 1280 x 720 4 samples 1596, 1622
+//                              (99,800); 1920 x 1080 4 samples 3134, 2768 (224,000)
+// disk lights:
+//   262k            640 x 360  8 samples 586, 538 (57,400)
+//   1M              640 x 360  8 samples 752, 812 (45,100), 16 samples 1118, 1052
+//                              (90,200); 853 x 479 8 samples 1098, 1088 (80,000)
+//   4M              640 x 360  8 samples 985, 1260 (49,900); 960 x 540 8 samples
+//                              1873, 2024 (112,000); 1280 x 720 4 samples 1839,
+//                              2169 (99,800), 16 samples 5409, 4424 (399,000)
+// tris: the scene's, 0 for several scenes.
+HR_RULE uint32_t packets_from(uint32_t samples, uint32_t tris, bool scattered) {
+    const uint32_t grain = tris >> (scattered ? 19 : 21), per = samples < 16u ? samples : 16u;
+    return ((grain > 1u ? grain : 1u) * (1u << 18) + per - 1u) / per;
+}
+
 }  // namespace hr

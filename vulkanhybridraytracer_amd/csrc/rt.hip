@@ -469,17 +469,18 @@ struct RtItems {
     }
 };
 
-// as k_shadows_spl: packets, or a walk per lane for the short lists of later depths
+// as k_shadows_spl: packets from `packets` waves of items on, a walk per lane for
+// the short lists of later depths
 template <bool OFF32>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void k_rt_shadows(
-    DevScene S, FrameArgs F, RtWork w, uint32_t lg2s, uint32_t nS, uint32_t depth, uint32_t* next_item,
-    unsigned long long* counters) {
+    DevScene S, FrameArgs F, RtWork w, uint32_t lg2s, uint32_t nS, uint32_t depth, uint32_t packets,
+    uint32_t* next_item, unsigned long long* counters) {
     __shared__ uint32_t stk[STACK_LDS * BLOCK];
     Cnt c = {};
     const uint32_t nh = w.cnt[2];
     RtItems src{F, w.hpos, w.hnrm, w.hpix, w.glist, w.bits, nh, lg2s, nS, depth, S.nodes4, S.tris, S.node_count};
     const uint32_t nitems = w.cnt[3] << lg2s;
-    if (list_packets(nitems, 1u << lg2s)) packet_loop(src, nitems, next_item, c);
+    if ((nitems >> 6) >= packets) packet_loop(src, nitems, next_item, c);
     else item_loop<OFF32>(src, nitems, next_item, stk + threadIdx.x, c);
     flush_counters(c, counters, false);
 }
@@ -597,6 +598,7 @@ hipError_t launch_rt_wavefront(const DevScene& s, const FrameArgs& f, float4* ac
     const uint32_t spp = max(f.spp, 1u);
     const uint32_t gmax = f.nl * P;  // (light, hit) groups of a depth at most
     const GroupListTail gt = group_list_tail(w.gtail, gmax);
+    const uint32_t packets = packets_from(1u << lg2s, s.tri_count, scattered_lights(f));
     for (uint32_t nS = 0; nS < spp; ++nS) {
         k_rt_begin<<<nbT, BLOCK, 0, st>>>(f, w, nS);
         for (uint32_t depth = 0; depth < f.max_depth; ++depth) {
@@ -615,9 +617,11 @@ hipError_t launch_rt_wavefront(const DevScene& s, const FrameArgs& f, float4* ac
                 scan_and_scatter(gmax, gt, w.cnt + 3, w.glist, st);
             }
             if ((uint64_t)s.wide_count * sizeof(TNode4) <= 0xFFFFFFFFull)
-                k_rt_shadows<true><<<resident_blocks, BLOCK, 0, st>>>(s, f, w, lg2s, nS, depth, next_item, counters);
+                k_rt_shadows<true><<<resident_blocks, BLOCK, 0, st>>>(s, f, w, lg2s, nS, depth, packets, next_item,
+                                                                      counters);
             else
-                k_rt_shadows<false><<<resident_blocks, BLOCK, 0, st>>>(s, f, w, lg2s, nS, depth, next_item, counters);
+                k_rt_shadows<false><<<resident_blocks, BLOCK, 0, st>>>(s, f, w, lg2s, nS, depth, packets, next_item,
+                                                                       counters);
             k_rt_shade<<<nbT, BLOCK, 0, st>>>(s, f, w, lg2s, nS, depth);
         }
         k_rt_end<<<nbP, BLOCK, 0, st>>>(f, w, nS, accum, frame_signed);

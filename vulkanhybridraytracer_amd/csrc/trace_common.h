@@ -1324,17 +1324,6 @@ __device__ __forceinline__ void packet_loop(Src& src, uint32_t nitems, uint32_t*
     }
 }
 
-// Packets (packet_loop) or a walk per lane (item_loop) for nitems items of
-// `samples` per (surface point, light)? Packets need waves to hide their serial
-// node loads behind, and rays that stay together; rays of one point do. With
-// 4 lights (us, per lane and as packets): 320 x 180, 4 samples (7,200 packets
-// with rays) 252, 295; 640 x 360, 4 samples (28,800) 390, 393; 8 samples (57,600)
-// 552, 500; 320 x 180, 16 samples (28,800) 360, 340; 1280 x 720, 4 samples
-// (115,000) 963, 786; 16 samples (460,000) 2710, 1910.
-__device__ __forceinline__ bool list_packets(uint32_t nitems, uint32_t samples) {
-    return (uint64_t)(nitems >> 6) * min(samples, 16u) >= (1u << 18);
-}
-
 // the number of set bits of a group's item window (stride 2^lg2s, lg2s <= 6):
 // whole words for 32 and 64, a masked part of one word below (a shift by 32
 // would not give a full mask)
