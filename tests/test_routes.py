@@ -72,3 +72,12 @@ def test_packets_ask_for_more_waves_in_fine_scenes(rule):
              (3, 0, 0, 87_381, 0), (3, 0, 0, 87_382, 1), (64, 0, 0, 16_384, 1), (64, 0, 1, 16_383, 0)]
     got = rule(*["%du >= packets_from(%du, %du, %d)" % (w, s, t, d) for s, t, d, w, _ in cases])
     assert got == [e for *_, e in cases]
+
+
+def test_lanes_of_bare_ray_queries(rule):
+    """few rays over many waves, and counts near 2^32 as any other: their sums would wrap"""
+    cases = [(1, 2), (4_096, 2), (40_960, 10), (98_305, 25), (262_143, 64), (2 ** 32 - 4_096, 64), (2 ** 32 - 4_095, 64),
+             (2 ** 32 - 1, 64)]
+    assert rule(*["ray_lanes(%du)" % n for n, _ in cases]) == [e for _, e in cases]
+    assert rule("ray_queue(262143u, 1000000u)", "ray_queue(262144u, 100000u)", "ray_queue(4000000u, 99999u)") == [0, 1, 0]
+    assert rule("div_up(4294967295u, 256u)", "div_up(256u, 256u)", "div_up(0u, 8u)") == [2 ** 24, 1, 0]

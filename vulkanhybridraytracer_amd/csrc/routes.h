@@ -128,4 +128,23 @@ HR_RULE uint32_t packets_from(uint32_t samples, uint32_t tris, bool scattered) {
     return ((grain > 1u ? grain : 1u) * (1u << 18) + per - 1u) / per;
 }
 
+HR_RULE uint32_t div_up(uint32_t a, uint32_t b) { return a / b + (a % b != 0u ? 1u : 0u); }
+
+// Bare ray queries (us before and now; closest hits). As a queue, whose lanes take
+// new rays, or a ray per lane? 4.1M rays, 1M triangles: 2415 -> 1641, any hit 1458
+// -> 1090; in small scenes a ray is over before its lane's next one is fetched
+// (80k triangles, 1M rays: 245 -> 275, 20k: 135 -> 211).
+HR_RULE bool ray_queue(uint32_t rays, uint32_t tris) { return rays >= 262144u && tris >= LARGE_SCENE; }
+// With a ray per lane, the lanes of a wave in use: the rays go over about 4096
+// waves, 2 a wave at least, since a wave takes as long as the nodes its rays visit
+// together (4,096 random pixels of a 20k-triangle scene 42 -> 28, of a 1M-triangle
+// one 207 -> 84; 16 lanes at least: 36 and 142). From 120,000 rays to 262,144 full
+// waves are as good within 10% either way (131,072 rays, full and partly used: 20k
+// triangles 44, 47, 16k 142, 128; 200,000 rays: 46, 49 and 145, 142, 1M any hit
+// 218, 199).
+HR_RULE uint32_t ray_lanes(uint32_t rays) {
+    const uint32_t lanes = div_up(rays, 4096u);
+    return lanes > 64u ? 64u : (lanes > 2u ? lanes : 2u);
+}
+
 }  // namespace hr
