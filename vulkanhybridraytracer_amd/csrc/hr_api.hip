@@ -77,6 +77,29 @@ struct SceneArena {
         return HR_OK;
     }
 };
+// Host arrays that follow one another on the device: put() each, then flush().
+// Arrays below SMALL are gathered and copied together, others from where they are:
+// a copy of its own is 10 us however short (4000 meshes of 11 KB loaded in 99 ms
+// when only their vertices went one by one, in 128 ms with their indices, now in 27).
+struct UploadRun {
+    static constexpr size_t SMALL = 64u << 10, RUN = 4u << 20;
+    char* dst;                // of the next array
+    std::vector<char> run;    // the gathered arrays before it
+    hipError_t flush() {
+        const hipError_t e = run.empty() ? hipSuccess
+                                         : hipMemcpy(dst - run.size(), run.data(), run.size(), hipMemcpyHostToDevice);
+        run.clear();
+        return e;
+    }
+    hipError_t put(const void* src, size_t bytes) {
+        hipError_t e = hipSuccess;
+        if (bytes >= SMALL || run.size() + bytes > RUN) e = flush();
+        if (e == hipSuccess && bytes >= SMALL) e = hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+        else if (bytes) run.insert(run.end(), static_cast<const char*>(src), static_cast<const char*>(src) + bytes);
+        dst += bytes;
+        return e;
+    }
+};
 // releases one buffer of s->allocs (device idle: the caller synchronised)
 void scene_free(hr_scene* s, void* p) {
     if (!p) return;
@@ -762,14 +785,14 @@ hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_c
         return st;
     }
     // uploads: vertices as-is (44-byte stride), indices as-is
-    for (uint32_t m = 0; m < mesh_count && he == hipSuccess; ++m) {
-        if (meshes[m].vertex_count)
-            he = hipMemcpy(s->d_verts + vbase[m] * sizeof(hr_vertex), meshes[m].vertices,
-                           (size_t)meshes[m].vertex_count * sizeof(hr_vertex), hipMemcpyHostToDevice);
-        if (he == hipSuccess && meshes[m].index_count)
-            he = hipMemcpy(s->d_indices + ibase[m], meshes[m].indices, (size_t)meshes[m].index_count * sizeof(uint32_t),
-                           hipMemcpyHostToDevice);
-    }
+    UploadRun up{reinterpret_cast<char*>(s->d_verts), {}};
+    for (uint32_t m = 0; m < mesh_count && he == hipSuccess; ++m)
+        he = up.put(meshes[m].vertices, (size_t)meshes[m].vertex_count * sizeof(hr_vertex));
+    if (he == hipSuccess) he = up.flush();
+    up.dst = reinterpret_cast<char*>(s->d_indices);
+    for (uint32_t m = 0; m < mesh_count && he == hipSuccess; ++m)
+        he = up.put(meshes[m].indices, (size_t)meshes[m].index_count * sizeof(uint32_t));
+    if (he == hipSuccess) he = up.flush();
     if (he == hipSuccess && prim_count)
         he = hipMemcpy(s->d_prims, s->h_prims.data(), prim_count * sizeof(PrimInfo), hipMemcpyHostToDevice);
     if (he == hipSuccess && prim_count)
