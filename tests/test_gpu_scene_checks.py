@@ -47,3 +47,46 @@ def test_index_out_of_range(gpu_ctx, prim, corner):
                 int(p["first_index"]) + int(p["index_count"]) - 3 + corner < int(q["first_index"]) + int(q["index_count"]))
     assert "primitive %d: vertex index out of range" % first in _build_error(gpu_ctx, sc)
     hr.HybridScene(gpu_ctx, _two_meshes()).close()
+
+
+def _bad_vertex(sc):
+    sc.meshes[1][0][3, 0] = np.inf
+    return "mesh 1 vertex 3: non-finite"
+
+
+def _bad_index(prim):
+    def f(sc):
+        p = sc.prims[prim]
+        v, idx = sc.meshes[int(p["mesh"])]
+        idx[int(p["first_index"])] = len(v)
+        return "primitive %d: vertex index out of range" % prim
+    return f
+
+
+def _bad_material(prim):
+    def f(sc):
+        sc.prims["material"][prim] = len(sc.materials)
+        return "primitive %d: mesh, index range or material" % prim
+    return f
+
+
+def _bad_model(prim):
+    def f(sc):
+        sc.prims["model"][prim, 5] = np.nan
+        return "primitive %d: non-finite model" % prim
+    return f
+
+
+@pytest.mark.parametrize("faults", [(_bad_vertex, _bad_index(0)), (_bad_vertex, _bad_material(0)),
+                                    (_bad_vertex, _bad_model(0)), (_bad_index(0), _bad_material(1)),
+                                    (_bad_index(0), _bad_model(1)), (_bad_index(0), _bad_model(0)),
+                                    (_bad_material(0), _bad_index(1)), (_bad_model(0), _bad_index(1))],
+                         ids=["vertex-index", "vertex-material", "vertex-model", "index-material", "index-model",
+                              "index-model of one", "material-index", "model-index"])
+def test_the_first_of_two_faults_is_named(gpu_ctx, faults):
+    """meshes come before primitives, an earlier primitive before a later one"""
+    sc = _two_meshes()
+    sc.prims = sc.prims.copy()
+    assert int(sc.prims["mesh"][0]) != int(sc.prims["mesh"][1])
+    want = [f(sc) for f in faults][0]
+    assert want in _build_error(gpu_ctx, sc)

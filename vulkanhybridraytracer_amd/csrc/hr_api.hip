@@ -667,6 +667,43 @@ void hr_scene_destroy(hr_scene* s) {
     delete s;
 }
 
+// The first fault of a scene's arrays, of the meshes and then of the primitives.
+// geometry: also the positions' and indices' (9 ms for 1.8M vertices; hr_scene_build
+// leaves these to the GPU and comes back for the fault's name).
+static hr_status check_scene(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_count, const hr_primitive* prims,
+                             uint32_t prim_count, uint32_t material_count, bool geometry) {
+    uint64_t nv = 0, ni = 0, tri = 0;
+    for (uint32_t m = 0; m < mesh_count; ++m) {
+        if ((meshes[m].vertex_count && !meshes[m].vertices) || (meshes[m].index_count && !meshes[m].indices))
+            return fail(ctx, HR_E_INVALID, "mesh %u: NULL arrays", m);
+        nv += meshes[m].vertex_count;
+        ni += meshes[m].index_count;
+        for (uint32_t v = 0; geometry && v < meshes[m].vertex_count; ++v) {
+            const float* p = meshes[m].vertices[v].position;
+            if (!std::isfinite(p[0]) || !std::isfinite(p[1]) || !std::isfinite(p[2]))
+                return fail(ctx, HR_E_INVALID, "mesh %u vertex %u: non-finite position", m, v);
+        }
+    }
+    if (nv >= 0xFFFFFFFFull || ni >= 0xFFFFFFFFull) return fail(ctx, HR_E_UNSUPPORTED, "too many vertices or indices");
+    for (uint32_t i = 0; i < prim_count; ++i) {
+        const hr_primitive& hp = prims[i];
+        if (hp.mesh >= mesh_count || hp.index_count % 3 != 0 ||
+            (uint64_t)hp.first_index + hp.index_count > meshes[hp.mesh].index_count || hp.material < 0 ||
+            (uint32_t)hp.material >= material_count)
+            return fail(ctx, HR_E_INVALID, "primitive %u: mesh, index range or material out of range", i);
+        const hr_mesh& mh = meshes[hp.mesh];
+        for (uint32_t k = 0; geometry && k < hp.index_count; ++k)
+            if (mh.indices[hp.first_index + k] >= mh.vertex_count)
+                return fail(ctx, HR_E_INVALID, "primitive %u: vertex index out of range", i);
+        for (int k = 0; k < 16; ++k)
+            if (!std::isfinite(hp.model[k])) return fail(ctx, HR_E_INVALID, "primitive %u: non-finite model matrix", i);
+        tri += hp.index_count / 3;
+    }
+    if (tri >= MAX_TRIS)
+        return fail(ctx, HR_E_UNSUPPORTED, "%llu triangles exceed the 2^27 limit", (unsigned long long)tri);
+    return HR_OK;
+}
+
 hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_count, const hr_primitive* prims,
                          uint32_t prim_count, const hr_material* materials, uint32_t material_count,
                          const hr_build_params* params, hr_scene** out) {
@@ -680,16 +717,18 @@ hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_c
     if (leaf_max > LEAF_MAX_LIMIT) return fail(ctx, HR_E_INVALID, "leaf_max %u exceeds %u", leaf_max, LEAF_MAX_LIMIT);
     for (uint32_t i = 0; i < material_count; ++i) HR_TRY(check_material(ctx, materials[i], i, material_count));
 
+    const hr_status table = check_scene(ctx, meshes, mesh_count, prims, prim_count, material_count, false);
+    if (table != HR_OK) {  // a fault of the geometry may come before it
+        const hr_status fault = check_scene(ctx, meshes, mesh_count, prims, prim_count, material_count, true);
+        return fault != HR_OK ? fault : table;
+    }
+
     // concatenated vertices / indices with per-mesh bases
     std::vector<uint64_t> vbase(mesh_count + 1, 0), ibase(mesh_count + 1, 0);
     for (uint32_t m = 0; m < mesh_count; ++m) {
-        if ((meshes[m].vertex_count && !meshes[m].vertices) || (meshes[m].index_count && !meshes[m].indices))
-            return fail(ctx, HR_E_INVALID, "mesh %u: NULL arrays", m);
         vbase[m + 1] = vbase[m] + meshes[m].vertex_count;
         ibase[m + 1] = ibase[m] + meshes[m].index_count;
     }
-    if (vbase[mesh_count] >= 0xFFFFFFFFull || ibase[mesh_count] >= 0xFFFFFFFFull)
-        return fail(ctx, HR_E_UNSUPPORTED, "too many vertices or indices");
 
     hr_scene* s = new hr_scene();
     s->ctx = ctx;
@@ -704,19 +743,7 @@ hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_c
     s->h_prim_tri_offset.resize(prim_count + 1);
     for (uint32_t i = 0; i < prim_count; ++i) {
         const hr_primitive& hp = prims[i];
-        if (hp.mesh >= mesh_count || hp.index_count % 3 != 0 ||
-            (uint64_t)hp.first_index + hp.index_count > meshes[hp.mesh].index_count || hp.material < 0 ||
-            (uint32_t)hp.material >= material_count) {
-            hr_scene_destroy(s);
-            return fail(ctx, HR_E_INVALID, "primitive %u: mesh, index range or material out of range", i);
-        }
         const hr_mesh& mh = meshes[hp.mesh];
-        for (int k = 0; k < 16; ++k) {
-            if (!std::isfinite(hp.model[k])) {
-                hr_scene_destroy(s);
-                return fail(ctx, HR_E_INVALID, "primitive %u: non-finite model matrix", i);
-            }
-        }
         PrimInfo& p = s->h_prims[i];
         memset(&p, 0, sizeof(p));
         p.tri_offset = (uint32_t)tri;
@@ -728,10 +755,6 @@ hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_c
         memcpy(&s->h_models[(size_t)i * 16], hp.model, 16 * sizeof(float));
         s->h_prim_tri_offset[i] = (uint32_t)tri;
         tri += hp.index_count / 3;
-    }
-    if (tri >= MAX_TRIS) {
-        hr_scene_destroy(s);
-        return fail(ctx, HR_E_UNSUPPORTED, "%llu triangles exceed the 2^27 limit", (unsigned long long)tri);
     }
     s->h_prim_tri_offset[prim_count] = (uint32_t)tri;
     s->ntri = (uint32_t)tri;
@@ -780,10 +803,13 @@ hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_c
     arena.add(&b.tri_prim, n);
     arena.add(&b.depth, 1);
     check(arena.allocate(s));
-    if (st != HR_OK) {
+    // of a scene that cannot be had and is wrong, what is wrong is named
+    auto refused = [&](hr_status other) {
         hr_scene_destroy(s);
-        return st;
-    }
+        const hr_status fault = check_scene(ctx, meshes, mesh_count, prims, prim_count, material_count, true);
+        return fault != HR_OK ? fault : other;
+    };
+    if (st != HR_OK) return refused(st);
     // uploads: vertices as-is (44-byte stride), indices as-is
     UploadRun up{reinterpret_cast<char*>(s->d_verts), {}};
     for (uint32_t m = 0; m < mesh_count && he == hipSuccess; ++m)
@@ -802,10 +828,7 @@ hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_c
                        hipMemcpyHostToDevice);
     if (he == hipSuccess)
         he = hipMemcpy(s->d_mats, materials, material_count * sizeof(hr_material), hipMemcpyHostToDevice);
-    if (he != hipSuccess) {
-        hr_scene_destroy(s);
-        return hip_fail(ctx, he, "scene upload");
-    }
+    if (he != hipSuccess) return refused(hip_fail(ctx, he, "scene upload"));
     b.verts = s->d_verts;
     b.indices = s->d_indices;
     b.prims = s->d_prims;
@@ -815,23 +838,12 @@ hr_status hr_scene_build(hr_context* ctx, const hr_mesh* meshes, uint32_t mesh_c
     b.tri_count = n;
     b.leaf_max = leaf_max;
 
-    // non-finite positions and indices out of range (first of each), and the
-    // normals as float4 (the rtVertexAttribute repack of renderer.cpp:3018-3048)
-    uint32_t bad[2];
-    he = lbvh_check(b, s->d_vnormal, (uint32_t)nv, bad, ctx->stream);
-    if (he != hipSuccess) {
-        hr_scene_destroy(s);
-        return hip_fail(ctx, he, "scene check");
-    }
-    if (bad[0] != 0xFFFFFFFFu) {
-        const uint32_t m = (uint32_t)(std::upper_bound(vbase.begin(), vbase.end(), (uint64_t)bad[0]) - vbase.begin()) - 1u;
-        hr_scene_destroy(s);
-        return fail(ctx, HR_E_INVALID, "mesh %u vertex %u: non-finite position", m, (uint32_t)(bad[0] - vbase[m]));
-    }
-    if (bad[1] != 0xFFFFFFFFu) {
-        hr_scene_destroy(s);
-        return fail(ctx, HR_E_INVALID, "primitive %u: vertex index out of range", bad[1]);
-    }
+    // non-finite positions and indices out of range, and the normals as float4
+    // (the rtVertexAttribute repack of renderer.cpp:3018-3048)
+    uint32_t bad = 0;
+    he = lbvh_check(b, s->d_vnormal, (uint32_t)nv, &bad, ctx->stream);
+    if (he != hipSuccess) return refused(hip_fail(ctx, he, "scene check"));
+    if (bad) return refused(fail(ctx, HR_E_INVALID, "non-finite position or vertex index out of range"));
 
     he = hipEventRecord(ctx->ev[0], ctx->stream);
     if (he == hipSuccess) he = lbvh_build(b, ctx->stream, !(ctx->tuning.bvh_flags & HR_BVH_NO_TREELETS));

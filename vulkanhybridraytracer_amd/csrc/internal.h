@@ -280,10 +280,9 @@ struct BuildBuffers {
     uint32_t* depth;    // 1 uint
 };
 size_t radix_hist_words(uint32_t n);
-// The uploaded geometry checked: bad[0] the first vertex (of the concatenated
-// ones) with a non-finite position, bad[1] the first primitive with an index
-// beyond its mesh, 0xFFFFFFFF: none (waits for the stream). Also writes vnormal,
-// the vertices' normals (xyz, 0).
+// The uploaded geometry checked: *bad is set to 1 by a non-finite position or an
+// index beyond its mesh, else 0 (waits for the stream). Also writes vnormal, the
+// vertices' normals (xyz, 0).
 hipError_t lbvh_check(const BuildBuffers& b, float4* vnormal, uint32_t vertex_count, uint32_t* bad, hipStream_t st);
 // full build in two calls: lbvh_build makes the binary tree and chooses the
 // 4-wide nodes (sets wide_count, synchronising the stream); the caller then

@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void k_check_vertices(const uint8_t* verts, ui
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float* v = (const float*)(verts + (size_t)i * 44u);
-    if (!(isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]))) atomicMin(bad, i);
+    if (!(isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]))) *bad = 1u;
     vnormal[i] = make_float4(v[3], v[4], v[5], 0.0f);
 }
 __global__ __launch_bounds__(256) void k_check_indices(BuildBuffers b, uint32_t* bad) {
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void k_check_indices(BuildBuffers b, uint32_t*
     const uint32_t p = find_prim(b.prim_tri_offset, b.prim_count, g);
     const PrimInfo& pi = b.prims[p];
     const uint32_t* idx = b.indices + pi.index_base + 3u * (g - pi.tri_offset);
-    if (max(max(idx[0], idx[1]), idx[2]) >= pi.vertex_count) atomicMin(bad + 1, p);
+    if (max(max(idx[0], idx[1]), idx[2]) >= pi.vertex_count) *bad = 1u;
 }
 
 // World triangles, their boxes and primitives; with_bounds: also the bounds of
@@ -1158,13 +1158,13 @@ hipError_t choose_wide(BuildBuffers& b, hipStream_t st) {
 size_t radix_hist_words(uint32_t n) { return 256u * (size_t)blocks(n > 0 ? n : 1, RS_TILE); }
 
 hipError_t lbvh_check(const BuildBuffers& b, float4* vnormal, uint32_t vertex_count, uint32_t* bad, hipStream_t st) {
-    uint32_t* d_bad = b.bounds + 6;  // the words after the centre bounds
-    k_fill_u32<<<1, 64, 0, st>>>(d_bad, 2u, 0xFFFFFFFFu);
+    uint32_t* d_bad = b.bounds + 6;  // the word after the centre bounds
+    k_fill_u32<<<1, 64, 0, st>>>(d_bad, 1u, 0u);
     if (vertex_count)
         k_check_vertices<<<blocks(vertex_count, 256), 256, 0, st>>>(b.verts, vertex_count, vnormal, d_bad);
     if (b.tri_count) k_check_indices<<<blocks(b.tri_count, 256), 256, 0, st>>>(b, d_bad);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(bad, d_bad, 2u * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(bad, d_bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     return e;
 }
