@@ -23,6 +23,17 @@ def rule(tmp_path_factory):
     return run
 
 
+def test_dealt_queue_covers_every_ray(rule):
+    """any queue that the grid's lanes hold, on small and large grids; short rays over fewer waves"""
+    cases = [(n, w, t) for w in (1, 4, 100, 4095, 4096, 4097, 8192) for t in (20_000, 1_000_000)
+             for n in sorted({1, 15, 16 * w, 17 * w + 1, 64 * w - 1, 64 * w, min(64 * w, 262_145)}) if 1 <= n <= 64 * w]
+    got = rule(*["dealt_lanes(%du, %du, %du)" % c for c in cases])
+    for (n, w, t), per in zip(cases, got):
+        assert 16 <= per <= 64 and w * per >= n, (n, w, t, per)
+    assert rule("dealt_lanes(200000u, 8192u, 20000u)", "dealt_lanes(200000u, 8192u, 1000000u)",
+                "dealt_lanes(500000u, 8192u, 20000u)", "dealt_lanes(1u, 8192u, 20000u)") == [49, 25, 64, 16]
+
+
 def test_dealt_queue_walks_with_part_of_its_own_lanes(rule):
     """a wave leaves the node loop for its leaves only when a share of the lanes
     it holds has one, also where it holds few"""

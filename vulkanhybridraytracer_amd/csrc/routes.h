@@ -13,7 +13,28 @@
 
 namespace hr {
 
-// Ray queues (consume_queue). Lanes of a wave stay in the inner node loop until
+HR_RULE uint32_t div_up(uint32_t a, uint32_t b) { return a / b + (a % b != 0u ? 1u : 0u); }
+
+// Triangles from which a scene's rays are long: they visit many nodes and their
+// data leaves the caches, so idle lanes and single launches cost less than walks
+// that wait for one another.
+constexpr uint32_t LARGE_SCENE = 100000u;
+
+// Ray queues (consume_queue). A queue that the grid's lanes hold at once is dealt
+// out without take counters (finding all 8 bands empty costs every wave 8 round
+// trips to memory): so many rays to each of `waves` waves, 16 at least, the rest
+// of the lanes idle, since a wave takes as long as the nodes its rays visit
+// together. (640 x 360, depth 8: the 16 trace launches 985 -> 325 us; 853 x 479:
+// 1000 -> 817 us. 8 or 64 lanes a wave are no better.) In small scenes, whose rays
+// are short, over at most 4096 waves: 960 x 540, 20k triangles, us of the shading
+// pass (2 samples, 3 bounces) and of pure ray tracing (1 sample, 2 depths) over
+// all 8192 waves and 4096: 488, 448 and 719, 682 (657 with a ray per lane), 16k
+// triangles 998, 994 and 1274, 1228; but 1M triangles 1678, 1686 and 1719, 1776.
+HR_RULE uint32_t dealt_lanes(uint32_t rays, uint32_t waves, uint32_t tris) {
+    const uint32_t lanes = div_up(rays, tris < LARGE_SCENE && waves > 4096u ? 4096u : waves);
+    return lanes < 16u ? 16u : (lanes > 64u ? 64u : lanes);
+}
+// Lanes of a wave stay in the inner node loop until
 // fewer than this many of them walk; the others wait with a leaf or, in a queue
 // that hands out rays as lanes finish, without a ray. `live`: lanes of the wave
 // that hold a ray. A dealt queue (a ray per lane, none to take afterwards) has
@@ -26,11 +47,6 @@ namespace hr {
 //   256 x 256, 1M triangles    2358 / 2373 / 2242
 //   1280 x 720, 1M triangles   4448 / 3467 / 3303
 HR_RULE uint32_t queue_leave_below(bool dealt, uint32_t live) { return dealt ? live * 3u / 4u : 16u; }
-
-// Triangles from which a scene's rays are long: they visit many nodes and their
-// data leaves the caches, so idle lanes and single launches cost less than walks
-// that wait for one another.
-constexpr uint32_t LARGE_SCENE = 100000u;
 
 // Adaptive shadow passes in stages over the listed groups (powers of two up to
 // 64), or a lane per group? With 1 or 2 samples there is one stage and nothing to
@@ -127,8 +143,6 @@ HR_RULE uint32_t packets_from(uint32_t samples, uint32_t tris, bool scattered) {
     const uint32_t grain = tris >> (scattered ? 19 : 21), per = samples < 16u ? samples : 16u;
     return ((grain > 1u ? grain : 1u) * (1u << 18) + per - 1u) / per;
 }
-
-HR_RULE uint32_t div_up(uint32_t a, uint32_t b) { return a / b + (a % b != 0u ? 1u : 0u); }
 
 // Bare ray queries (us before and now; closest hits). As a queue, whose lanes take
 // new rays, or a ray per lane? 4.1M rays, 1M triangles: 2415 -> 1641, any hit 1458

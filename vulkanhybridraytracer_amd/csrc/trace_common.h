@@ -614,18 +614,13 @@ __device__ __forceinline__ uint32_t band_take(uint32_t* next, uint32_t n, uint32
 // ray; when its ray finishes it takes the next index (band_take over the
 // SHADOW_QUEUES band counters at `next`), so lanes do not wait for the
 // slowest ray of the wave. A queue that the grid's lanes hold at once is dealt
-// out without the counters (finding all 8 bands empty costs every wave 8 round
-// trips to memory), over as many waves as there are: QUEUE_LANES or more rays
-// a wave, the rest of its lanes idle, since a wave takes as long as the
-// nodes its rays visit together. (640 x 360, depth 8: the 16 trace launches 985
-// -> 325 us; 853 x 479: 1000 -> 817 us. 8 or 64 lanes a wave are no better.) Per ray the walk is the shared
+// out without the counters (dealt_lanes). Per ray the walk is the shared
 // near-first stack traversal (same order and counts as traverse()).
 //   get(i, o, d, tmin, tmax) -> false for an empty queue entry (skipped)
 //   put(i, hit, HitD)         result of entry i
-constexpr uint32_t QUEUE_LANES = 16u;
 template <bool ANY, bool COUNT, bool DEALT, class GetRay, class PutHit>
-__device__ __forceinline__ void consume_queue(const DevScene& S, uint32_t n, uint32_t* next, uint32_t* lds, Cnt& c, GetRay get,
-                             PutHit put) {
+__device__ __forceinline__ void consume_queue(const DevScene& S, uint32_t n, uint32_t* next, uint32_t* lds, Cnt& c,
+                                              GetRay get, PutHit put) {
     uint32_t cur = DONE, idx = 0;
     bool have = false;
     RayP r;
@@ -644,7 +639,7 @@ __device__ __forceinline__ void consume_queue(const DevScene& S, uint32_t n, uin
     uint32_t emptied = 0;
     uint32_t mine = n;  // DEALT: this lane's ray
     if (DEALT) {
-        const uint32_t waves = gridDim.x * (BLOCK / 64u), per = max((n + waves - 1u) / waves, QUEUE_LANES);
+        const uint32_t per = dealt_lanes(n, gridDim.x * (BLOCK / 64u), S.tri_count);
         const uint32_t wave = xcd_remap(blockIdx.x, gridDim.x) * (BLOCK / 64u) + (threadIdx.x >> 6);
         if ((threadIdx.x & 63u) < per) mine = wave * per + (threadIdx.x & 63u);
     }
