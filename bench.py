@@ -9,14 +9,16 @@ lights with 16 stratified shadow samples each, GGX glossy reflections at
 second of the K timed steps; primary rays (the G-buffer) are excluded.
 
 roofline: the shadow kernel (most of the rays) against the unit that binds
-it, VALU issue for packets (one wave64 instruction per SIMD every 4 cycles) or
-the vector-memory address path for walks per lane (256 CUs x 2.4 GHz / 16
-cycles: a CU's texture addresser takes 4 lanes per clock): its instructions per
-launch (rocprofv3, from the committed profile of the same workload) over its
-average launch time measured live with HIP events on the library's stream.
-Beside it: the
-measured TA busy fraction and VALU issue (a wave64 instruction per SIMD every
-4 cycles) with the lane utilisation, the algorithmic HBM bytes of the traced
+it, whichever is nearer to a rate that it cannot exceed: VALU issue (packets)
+at one wave64 instruction per SIMD every 2 cycles, or the vector-memory address
+path (walks per lane) at 256 CUs x 2.4 GHz / 16 cycles (a CU's texture addresser
+takes 4 lanes per clock). Adds, multiplies, FMAs, moves and integer adds issue
+every 2 cycles (8 waves per SIMD of one of them: 947 to 1078 Ginst/s), min, max
+and compares every 4 (571 to 593), so a mix of both ends below the peak. Its
+instructions per launch (rocprofv3, from the committed profile of the same
+workload) over its average launch time measured live with HIP events on the
+library's stream. Beside it: the measured TA busy fraction and VALU issue with
+the lane utilisation, the algorithmic HBM bytes of the traced
 rays (32 B per ray + 4 B per shadow hit + 32 B per binary node visited + 48 B
 per triangle tested, the counts from a counting launch that walks the oracle's
 order, outside the timed region) and the HBM bytes rocprofv3 measured, both
@@ -43,8 +45,8 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 # wave-level VALU issue peak of an MI355X: 256 CUs x 4 SIMDs x 2.4 GHz, one
-# wave64 VALU instruction per SIMD every 4 cycles
-VALU_PEAK_GINST = 256 * 4 * 2.4 / 4
+# wave64 VALU instruction per SIMD every 2 cycles
+VALU_PEAK_GINST = 256 * 4 * 2.4 / 2
 # wave-level vector memory instruction peak: a CU's texture addresser takes the
 # addresses of 4 lanes per clock, 16 clocks per 64-lane instruction
 VMEM_PEAK_GINST = 256 * 2.4 / 16
@@ -108,7 +110,7 @@ def roofline_of(kernel, workload, ms, rays, nodes, tris):
     traffic = prof.get("hbm_bytes_per_launch")
     vi = prof["valu_insts_per_launch"]
     valu = vi / (ms * 1e-3) / 1e9
-    # the unit nearer to its rate binds: packets issue VALU instructions and load
+    # the unit nearer to its peak binds: packets issue VALU instructions and load
     # through the scalar cache, the walks per lane load through the addresser
     if valu / VALU_PEAK_GINST >= ach / VMEM_PEAK_GINST:
         out.update(bound="valu_issue", achieved=round(valu, 1), peak=VALU_PEAK_GINST,

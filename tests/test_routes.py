@@ -92,3 +92,12 @@ def test_lanes_of_bare_ray_queries(rule):
     assert rule(*["ray_lanes(%du)" % n for n, _ in cases]) == [e for _, e in cases]
     assert rule("ray_queue(262143u, 1000000u)", "ray_queue(262144u, 100000u)", "ray_queue(4000000u, 99999u)") == [0, 1, 0]
     assert rule("div_up(4294967295u, 256u)", "div_up(256u, 256u)", "div_up(0u, 8u)") == [2 ** 24, 1, 0]
+
+
+def test_bench_binds_by_the_nearer_peak():
+    """no fraction of a bound above 1; packets by VALU issue, the walk per lane of the closest hits by vector loads"""
+    import bench
+    shadows = bench.roofline_of("k_shadows_spl", "hybrid_1080p_1m", 4.2, 57_000_000, 2_000_000_000, 300_000_000)
+    assert shadows["bound"] == "valu_issue" and 0.3 < shadows["frac"] < 1
+    trace = bench.roofline_of("k_wf_trace", "hybrid_1080p_4m", 13.2, 57_000_000, 2_000_000_000, 300_000_000)
+    assert trace["bound"] == "vmem" and trace["valu"]["issue_frac"] < trace["frac"] < 1
