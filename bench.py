@@ -69,13 +69,22 @@ def copy_probe(nbytes=1 << 30, reps=3):
     print(json.dumps({"copy_probe_bytes": nbytes, "reps": reps}), flush=True)
 
 
-def shadow_kernel_name(params):
-    """The kernel(s) of the timed shadow pass: sample-parallel for 4..64
-    samples (a power of two), in stages with adaptive sampling."""
-    if params["shadow_samples"] not in (4, 8, 16, 32, 64):
+def shadow_kernel_name(params, width, height, lights, tris):
+    """The kernel(s) of the timed shadow pass of one frame: the library's routes
+    (csrc/routes.h: adaptive_stages, shadow_route)."""
+    n, adaptive = params["shadow_samples"], bool(params.get("flags", 0) & 4)
+    groups = -(-width // 8) * -(-height // 8) * 64 * lights
+    lg2s = (n - 1).bit_length()
+    stages = n & (n - 1) == 0 and (n >= 4 or (n == 2 and tris >= 100000))
+    if n > 64 or (adaptive and not stages) or groups << lg2s >= 1 << 32:
         return "k_shadows"
-    if params.get("flags", 0) & 4:
+    if adaptive:
         return "k_shadows_spl (probe stage and later stages, with k_adaptive_decide)"
+    waves = groups << lg2s >> 6
+    if n <= 4 and tris < 100000 and waves < 16384:
+        return "k_shadows_once"
+    if tris < 500000 and (n == 1 and waves >= 49152 or n == 2 and tris >= 100000 and waves >= 98304):
+        return "k_shadows_direct"
     return "k_shadows_spl"
 
 
@@ -398,7 +407,7 @@ def main():
                                                                                   st_h.occluded_rays))
     W, H, nl = sc.width, sc.height, len(sc.lights)
     avg_shadow_ms = float(np.mean(ms_shadow))
-    kname = shadow_kernel_name(sc.params)
+    kname = shadow_kernel_name(sc.params, W, H, nl, sc.tri_count)
     roofline = roofline_of(kname.split()[0], sc.name, avg_shadow_ms, shadow_rays, shadow_nodes, shadow_tris)
     if kname != roofline["kernel"]:
         roofline["kernels"] = kname

@@ -94,6 +94,24 @@ def test_lanes_of_bare_ray_queries(rule):
     assert rule("div_up(4294967295u, 256u)", "div_up(256u, 256u)", "div_up(0u, 8u)") == [2 ** 24, 1, 0]
 
 
+def test_bench_names_the_routes(rule):
+    """bench.py's kernel names against the library's rules, over sample counts, sizes and scenes"""
+    import bench
+    frames = [(n, ad, w, h, nl, t) for n in (1, 2, 3, 4, 5, 16, 48, 64, 65) for ad in (0, 1)
+              for w, h, nl, t in ((97, 64, 2, 20_482), (640, 360, 2, 20_482), (1280, 720, 4, 262_144),
+                                  (1920, 1080, 4, 262_144), (1920, 1080, 4, 1_048_576), (16384, 16384, 4, 4_194_304))]
+    exprs = []
+    for n, ad, w, h, nl, t in frames:
+        groups = -(-w // 8) * -(-h // 8) * 64 * nl
+        exprs.append("%du > 64u || (%d && !adaptive_stages(%du, %du)) || ((uint64_t)%du << log2_up(%du)) >= (1ull << 32)"
+                     " ? 0u : (unsigned)shadow_route(%du, %d, %du, %du, true)"
+                     % (n, ad, n, t, groups, n, n, ad, groups, t))
+    names = ["k_shadows", "k_shadows_once", "k_shadows_direct", "k_shadows_spl"]
+    for (n, ad, w, h, nl, t), route in zip(frames, rule(*exprs)):
+        got = bench.shadow_kernel_name(dict(shadow_samples=n, flags=4 * ad), w, h, nl, t)
+        assert got.split()[0] == names[route], (n, ad, w, h, nl, t)
+
+
 def test_bench_binds_by_the_nearer_peak():
     """no fraction of a bound above 1; packets by VALU issue, the walk per lane of the closest hits by vector loads"""
     import bench
