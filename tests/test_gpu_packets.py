@@ -36,8 +36,9 @@ def _shadows(rd, flags):
     return rd.download_shadow(), int(st.shadow_rays), int(st.occluded_rays)
 
 
-# sizes: below every packet threshold; packets from 8 or 16 samples on; packets
-# for all counts (979 and 603: the right and bottom tiles are cut)
+# sizes: below every line for packets; packets from 8 or 16 samples on; packets
+# for 3 to 32 samples and the adaptive stages (979 and 603: the right and bottom
+# tiles are cut). 33 and 64 samples keep the walk per lane at every size.
 @pytest.mark.parametrize("kind", ["terrain", "spheres"])
 @pytest.mark.parametrize("w,h", [(45, 27), (322, 181), (979, 603)])
 @pytest.mark.parametrize("samples,adaptive", [(1, False), (2, False), (3, False), (4, False), (7, False), (16, False),

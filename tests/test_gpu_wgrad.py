@@ -55,3 +55,38 @@ def test_gradients_of_repeated_images(gpu_ctx, count):
     # each image's gradient carries the scale 1 / count through BF16 roundings
     assert np.linalg.norm(gn - g1) <= 2.0 ** -6 * np.linalg.norm(g1)
     dn.close()
+
+
+@pytest.mark.parametrize("count", [1, 16, 17, 33])
+def test_gradients_of_several_images(gpu_ctx, count):
+    """`count` different images (more than one launch takes from 17 on): the mean
+    loss and gradient are those of the single images"""
+    from vulkanhybridraytracer_amd import hr
+    r = np.random.default_rng(4)
+    h = w = 32
+    dn = denoise.Denoiser(gpu_ctx, seed=5)
+    keep, images, losses, grads = [], [], [], []
+    for k in range(count):
+        g = hr.GBuffer(gpu_ctx, w, h)
+        planes = {k2: r.uniform(0.1, 1.0, size=(h, w, 4)).astype(np.float32)
+                  for k2 in ("position", "normal", "albedo", "material", "emissive")}
+        g.upload(planes)
+        noisy, target = gpu_ctx.alloc(w * h * 16), gpu_ctx.alloc(w * h * 16)
+        noisy.upload(r.uniform(0, 0.5 + 0.2 * k, size=(h, w, 4)).astype(np.float32))
+        target.upload(r.uniform(0, 2, size=(h, w, 4)).astype(np.float32))
+        keep.append((g, noisy, target))
+        images.append(denoise.Denoiser.image(g, noisy.ptr, target.ptr, None, (0.0, 0.0, 0.0)))
+        loss, grad = dn.gradients(images[-1:])
+        losses.append(loss)
+        grads.append(grad.astype(np.float64))
+    ln, gn = dn.gradients(images)
+    mean, size = np.mean(grads, axis=0), np.mean([np.linalg.norm(g) for g in grads])
+    assert abs(ln - np.mean(losses)) <= 1e-6 * ln
+    # each image's gradient carries the scale 1 / count through BF16 roundings
+    tol = 2.0 ** -6 * size
+    assert np.linalg.norm(gn - mean) <= tol
+    if count > 1:
+        # the loss shows an image taken twice for another, both show one taken for all
+        assert abs(np.mean(losses[:1] + losses[:-1]) - np.mean(losses)) > 1e-4 * ln
+        assert np.linalg.norm(grads[0] - mean) > 4 * tol
+    dn.close()
