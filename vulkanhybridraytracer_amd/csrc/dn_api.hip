@@ -802,7 +802,6 @@ hr_status hr_dn_conv3x3_backward(hr_context* ctx, const void* x, const void* dy,
     TmpLayer t;
     HR_TRY(tmp_layer(ctx, weight, nullptr, cin, cout, t));
     const LayerInt& li = t.li;
-    const uint32_t P = n * h * w;
     if (dx) {
         ConvArgs a{};
         a.in = static_cast<const __bf16*>(dy);

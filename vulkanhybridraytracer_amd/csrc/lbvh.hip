@@ -1017,8 +1017,7 @@ __global__ __launch_bounds__(256) void k_depth(BuildBuffers b) {
     uint32_t n = b.tri_count;
     uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t d = 0;
-    if (k >= n) {
-    } else if (n >= 2) {
+    if (k < n && n >= 2) {
         uint32_t a = b.lparent[k];
         for (uint32_t step = 0; step < 4096u; ++step) {
             uint32_t sz = b.klast[a] - b.kfirst[a] + 1;
@@ -1026,7 +1025,7 @@ __global__ __launch_bounds__(256) void k_depth(BuildBuffers b) {
             if (a == 0) break;
             a = b.kparent[a];
         }
-    } else {
+    } else if (k < n) {
         d = 1;
     }
     // one atomic per wave

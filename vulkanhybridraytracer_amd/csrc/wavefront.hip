@@ -18,7 +18,8 @@
 //   k_wf_resolve  per pixel: the samples' bounce factors summed in sample
 //                 order, lit = direct * refl + ambient + emissive
 //
-// Pushes are aggregated (one atomic per workgroup, ranks from prefix sums). Queue lengths stay in device memory and every stage runs a fixed
+// Pushes are aggregated (one atomic per workgroup, ranks from prefix sums).
+// Queue lengths stay in device memory and every stage runs a fixed
 // grid that strides over the current length, so a frame needs no host
 // synchronisation. Each path owns a result slot (pixel, sample), so the
 // output does not depend on queue order.
