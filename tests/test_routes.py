@@ -77,7 +77,7 @@ def test_packets_ask_for_more_waves_in_fine_scenes(rule):
     """waves of items (samples, triangles, scattered lights) measured at both sides of the line: as packets or not"""
     cases = [(16, 262_144, 0, 18_800, 1), (8, 262_144, 1, 57_400, 1), (4, 262_144, 0, 28_700, 0),
              (16, 1_048_576, 0, 29_600, 1), (8, 1_048_576, 0, 45_100, 1), (8, 1_048_576, 1, 45_100, 0),
-             (8, 1_048_576, 1, 80_000, 1), (16, 1_048_576, 1, 90_200, 1), (16, 4_194_304, 0, 33_100, 1),
+             (8, 1_048_576, 1, 80_000, 1), (16, 1_048_576, 1, 90_200, 1), (16, 4_194_304, 0, 33_100, 1), (12, 4_194_304, 0, 35_000, 1), (12, 4_194_304, 0, 21_845, 0), (32, 4_194_304, 0, 16_384, 1),
              (8, 4_194_304, 0, 49_900, 0), (4, 4_194_304, 0, 99_800, 0), (4, 4_194_304, 0, 224_000, 1),
              (8, 4_194_304, 1, 112_000, 0), (4, 4_194_304, 1, 99_800, 0), (16, 4_194_304, 1, 399_000, 1),
              (3, 0, 0, 87_381, 0), (3, 0, 0, 87_382, 1), (64, 0, 0, 16_384, 1), (64, 0, 1, 16_383, 0)]
