@@ -110,9 +110,8 @@ def roofline_of(kernel, workload, ms, rays, nodes, tris):
                                "per_ray": "32 B ray + 4 B hit + 32 B per binary node + 48 B per triangle",
                                "nodes_per_ray": round(nodes / max(rays, 1), 2),
                                "tris_per_ray": round(tris / max(rays, 1), 2)}}
-    if prof is None:
-        out.update(bound="hbm", achieved=out["hbm_algorithmic"]["achieved"], peak=HBM_PEAK_GBS, unit="GB/s",
-                   frac=out["hbm_algorithmic"]["frac"], traffic=None)
+    if prof is None:  # the algorithmic bytes are no bound: the caches serve most of them
+        out.update(bound=None, achieved=None, peak=None, unit=None, frac=None, traffic=None)
         return out
     vm = prof["vmem_read_insts_per_launch"]
     ach = vm / (ms * 1e-3) / 1e9
@@ -259,6 +258,9 @@ def denoise_measure(steps=3, log_fn=log):
            "roofline": {"bound": "mfma", "achieved": round(tflops, 2), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                         "frac": round(tflops / BF16_PEAK_TFLOPS, 4), "flops_per_frame": int(flops),
                         "kernel": "denoiser forward (k_conv + features + kernel prediction)"}}
+    # what speedup_vs_64spp is against: above 32 samples the library keeps the slower of its two shadow walks
+    res["shadow_walk_64spp"] = ("per lane; as packets the 64 spp frame takes about 10 ms less and the ratio is "
+                                "about 7.0 (55.5, 46.0 and 6.53 ms for 4 spp + denoise, one run)")
     log_fn("denoise", res)
     dn.close()
     ctx.close()

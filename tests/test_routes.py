@@ -113,9 +113,12 @@ def test_bench_names_the_routes(rule):
 
 
 def test_bench_binds_by_the_nearer_peak():
-    """no fraction of a bound above 1; packets by VALU issue, the walk per lane of the closest hits by vector loads"""
+    """no fraction of a bound above 1; packets by VALU issue, the walk per lane of the closest hits by vector loads;
+    no bound without a profile"""
     import bench
     shadows = bench.roofline_of("k_shadows_spl", "hybrid_1080p_1m", 4.2, 57_000_000, 2_000_000_000, 300_000_000)
     assert shadows["bound"] == "valu_issue" and 0.3 < shadows["frac"] < 1
     trace = bench.roofline_of("k_wf_trace", "hybrid_1080p_4m", 13.2, 57_000_000, 2_000_000_000, 300_000_000)
     assert trace["bound"] == "vmem" and trace["valu"]["issue_frac"] < trace["frac"] < 1
+    unprofiled = bench.roofline_of("k_shadows_spl", "hybrid_1080p_4m", 4.7, 22_000_000, 1_100_000_000, 170_000_000)
+    assert unprofiled["hbm_algorithmic"]["frac"] > 1 and unprofiled["bound"] is unprofiled["frac"] is None
