@@ -1122,7 +1122,7 @@ __device__ __forceinline__ bool intersect_kz(const RayP& r, float Sx, float Sy, 
 // vector load, where a walk per lane paid about 110 and seven 16-byte loads at
 // half the lanes and was held by the texture addresser (87% busy). On the
 // 1080p, 1M-triangle frame (4 lights of 16 samples) the shadow launch went
-// from 4.89e9 VALU and 1.95e8 vector load instructions in 6.7 ms to 2.84e9 and
+// from 4.89e9 VALU and 1.95e8 vector load instructions in 6.7 ms to 2.65e9 and
 // 6e6 in 4.0 ms. The scalar side has to stay short too: with the near-first
 // order from the lanes' own distances (readlanes and a scalar sort) and
 // 64-bit lane masks per child, 3.4e9 scalar instructions bound it at 6.5 ms;
