@@ -377,7 +377,8 @@ hr_status hr_shade_hybrid(hr_scene* scene, const hr_gbuffer* gb,
  * ties on t broken by the smaller triangle id. HR_TRACE_COUNT_VISITS walks the
  * binary nodes in the oracle's near-first order and counts node visits and
  * triangle tests into stats (a slower kernel); without it the 4-wide nodes
- * are walked. Both give the same hits. stats (may be NULL) receives the
+ * are walked. Both give the same closest hits; with HR_TRACE_ANY_HIT the same
+ * rays hit, some of them another occluder. stats (may be NULL) receives the
  * counts and the time of whichever kernel ran. */
 #define HR_TRACE_ANY_HIT 1u
 #define HR_TRACE_COUNT_VISITS 2u
