@@ -55,7 +55,9 @@ HR_RULE uint32_t queue_leave_below(bool dealt, uint32_t live) { return dealt ? l
 // sample 256 x 256 218, 72, 1280 x 720 667, 198, 2 samples 667, 198; 4 lights in
 // 1M triangles: 1 sample 960 x 540 772, 573, but 2 samples 640 x 360 507, 791
 // and 1920 x 1080 1660, 2453 (262k: 480, 581 and 1372, 1817; 16k: 432, 412 and
-// 950, 1068).
+// 950, 1068). The line by size gives up what the stages won in small terrains
+// (16k: 97 x 64 135, 200, 1280 x 720 535, 688, but 853 x 479 580, 490) for the
+// two- to threefold in scenes of spheres.
 HR_RULE bool adaptive_stages(uint32_t samples, uint32_t tris) {
     return samples >= 1u && samples <= 64u && (samples & (samples - 1u)) == 0u &&
            (samples >= 4u || (samples == 2u && tris >= LARGE_SCENE));
